@@ -162,9 +162,21 @@ __global__ __launch_bounds__(DB) void k_absmax(size_t n, const double* __restric
 
 // ---------------------------------------------------------------- GMRES kernels
 
-// restart: beta = ||r||, monitor check on the true residual, g = beta e_1
+// the power of two 2^-e with |v| 2^-e in [1, 2), within the normal range of T (1 for a
+// zero or an invalid v)
+template <typename T>
+__device__ __forceinline__ double pow2_inverse(double v)
+{
+    constexpr int lim = sizeof(T) == 8 ? 1000 : 100;
+    if (v == 0.0 || !finite(v)) return 1.0;
+    const int e = ilogb(v);
+    return ldexp(1.0, -(e < -lim ? -lim : e > lim ? lim : e));
+}
+
+// restart: beta = ||r||, monitor check on the true residual, g = beta e_1; first (may be
+// null): the power of two near 1 / beta
 template <typename T, typename S>
-__global__ void k_gm_start(dstate* st, const T* n4, double* g, int m, S* sig, double* hist)
+__global__ void k_gm_start(dstate* st, const T* n4, double* g, int m, S* sig, T* first, double* hist)
 {
     if (st->done) {
         st->stop = 1;
@@ -182,6 +194,7 @@ __global__ void k_gm_start(dstate* st, const T* n4, double* g, int m, S* sig, do
     g[0] = beta;
     for (int i = 1; i <= m; ++i) g[i] = 0.0;
     sig[0] = (S)(1.0 / beta);
+    if (first != nullptr) *first = (T)pow2_inverse<T>(beta);
 }
 
 __device__ __forceinline__ void apply_rot(double& dx, double& dy, double cs, double sn)
@@ -536,6 +549,13 @@ __global__ __launch_bounds__(DB) void k_gm_dgks(const T* __restrict__ part, unsi
 // refinement on 120 x 128 x 124 60.9 ms against 92.9 ms.  Same steps, same residuals.
 // The estimate of step j - 1 is known after the product z = A u of step j; a cycle that
 // stops there has formed one z that it does not use.
+//
+// Scale.  A product of two vectors must neither over- nor underflow where CGS2's (of the
+// basis with A q_j) do not, so u and z are kept near 1 and ||A|| by powers of two, which
+// change no significand.  V_0 is the residual as it is; step 0 takes z = A (f V_0) with
+// f = 2^-e near 1 / ||r|| (k_gm_start).  Its products also hold (z, z), so that
+// F = 2^e near ||A q_0|| is known, and every candidate is divided by F: with column j - 1
+// completed from such a candidate, s_i and alpha enter H times F.
 
 // Products of the k columns V_0 .. V_{k-1} with u (NV 1) or with u and z (NV 2), over
 // chunks of kpc <= 8 columns (blockIdx.y): slot NV i + v of the partials.  FP64 vectors
@@ -632,20 +652,23 @@ __global__ __launch_bounds__(DB) void k_gm_proj(size_t n, int k, int kpc, basis_
 // completed (Givens step, estimate, stop flag) and, unless the cycle ends (LAST, j = m),
 // column j of H and the coefficients of k_gm_next are formed.  Hq holds the columns of H
 // before the rotations, R after them.  coef: [0, j) of V_j, MAXB + [0, j) of u', then
-// u' takes coef[2 MAXB] z + coef[2 MAXB + 1] V_j.  One block: a wave per product for the
+// u' takes coef[2 MAXB] z + coef[2 MAXB + 1] V_j; coef[2 MAXB + 2] keeps F.  first is f of
+// step 0, whose products are those of V_0 and z.  One block: a wave per product for the
 // merges, then thread 0 runs the rotations while the waves after the first form column j.
-template <bool LAST>
+template <typename T, bool LAST>
 __global__ __launch_bounds__(1024) void k_gm_step(const double* __restrict__ part, unsigned G, int j,
                                                   double* __restrict__ Hq, double* __restrict__ R, int ldh,
                                                   double* __restrict__ cs, double* __restrict__ sn,
                                                   double* __restrict__ g, double* __restrict__ sig,
-                                                  double* __restrict__ coef, dstate* __restrict__ st)
+                                                  double* __restrict__ coef, const T* __restrict__ first,
+                                                  dstate* __restrict__ st)
 {
     if (st->stop) return;
     constexpr int NV = LAST ? 1 : 2;
     __shared__ double pr[2 * (MAXB + 1)];           // (V_i, u), (V_i, z); later s_i, r_i
     __shared__ double sg[MAXB], hcol[MAXB + 1], rot[MAXB + 1], lcs[MAXB], lsn[MAXB];
-    __shared__ double sca[3];                       // sig_j, t, alpha
+    __shared__ double fac;                          // F
+    __shared__ double sca[5];                       // sig_j, t, h_{j,j-1}, sig_j / f, 1 / F
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     if (tid < j) {
         sg[tid] = sig[tid];
@@ -653,7 +676,7 @@ __global__ __launch_bounds__(1024) void k_gm_step(const double* __restrict__ par
         lcs[tid] = tid + 1 < j ? cs[tid] : 0.0;
         lsn[tid] = tid + 1 < j ? sn[tid] : 0.0;
     }
-    const int slots = NV * (j + 1);
+    const int slots = NV * (!LAST && j == 0 ? 2 : j + 1);
     auto merge_slots = [&](auto nc) {   // a wave for N products at a time
         constexpr int N = decltype(nc)::value;
         for (int s0 = wid * N; s0 < slots; s0 += 16 * N) {
@@ -688,15 +711,30 @@ __global__ __launch_bounds__(1024) void k_gm_step(const double* __restrict__ par
         if (lane == 0) {
             const double a2 = s[j] - ss;
             const double al = a2 <= 0.0 ? 0.0 : sqrt(a2);   // a NaN stays one
-            const double sj = al != 0.0 ? 1.0 / al : 0.0;
+            double sj = al != 0.0 ? 1.0 / al : 0.0, zf, F;
+            if (j == 0) {
+                // ||r||^2 out of range: k_gm_start's 1 / ||r||
+                if (!(a2 >= 0x1p-900 && a2 <= 0x1p900) && g[0] != 0.0) sj = sig[0];
+                zf = sj / (double)*first;
+                const double zi = LAST ? 1.0 : pow2_inverse<double>(sqrt(r[1]) * zf);
+                F = 1.0 / zi;
+                sca[4] = zi;
+                coef[2 * MAXB + 2] = F;
+            } else {
+                zf = sj;
+                F = coef[2 * MAXB + 2];
+                sca[4] = 1.0 / F;
+            }
             sca[0] = sj;
             sca[1] = LAST ? 0.0 : (r[j] - sr) * sj;
-            sca[2] = al;
+            sca[2] = al * F;
+            sca[3] = zf;
+            fac = F;
         }
     }
     __syncthreads();
     if (tid < j) {
-        hcol[tid] += s[tid];
+        hcol[tid] = __builtin_fma(s[tid], fac, hcol[tid]);
         Hq[(size_t)(j - 1) * ldh + tid] = hcol[tid];
     }
     if (tid == 0 && j > 0) {
@@ -746,18 +784,18 @@ __global__ __launch_bounds__(1024) void k_gm_step(const double* __restrict__ par
     }
     if (!LAST && wid >= 1) {
         const int l = tid - 64;
-        const double sj = sca[0], t = sca[1];
+        const double sj = sca[0], t = sca[1], zf = sca[3], zi = sca[4];
         if (l < j) {
             double h = r[l];
             for (int i = l > 0 ? l - 1 : 0; i + 1 < j; ++i) h = __builtin_fma(-Hq[(size_t)i * ldh + l], s[i], h);
             h = __builtin_fma(-hcol[l], s[j - 1], h);
             Hq[(size_t)j * ldh + l] = h * sj;
             coef[l] = -s[l] * sg[l];
-            coef[MAXB + l] = -sj * r[l] * sg[l];
+            coef[MAXB + l] = -(sj * zi) * r[l] * sg[l];
         } else if (l == j) {
-            Hq[(size_t)j * ldh + j] = (j > 0 ? __builtin_fma(-hcol[j], s[j - 1], t) : t) * sj;
-            coef[2 * MAXB] = sj;
-            coef[2 * MAXB + 1] = -t * sj * sj;
+            Hq[(size_t)j * ldh + j] = (j > 0 ? __builtin_fma(-hcol[j], s[j - 1], t) : t) * zf;
+            coef[2 * MAXB] = zf * zi;
+            coef[2 * MAXB + 1] = -t * (zf * zi) * sj;
         }
     }
     __syncthreads();
@@ -1829,7 +1867,8 @@ private:
         DS_CHECK(sn.alloc(m));
         DS_CHECK(g.alloc(m + 1));
         DS_CHECK(n4.alloc(4));
-        DS_CHECK(dcoef.alloc(2 * MAXB + 2));
+        DS_CHECK(dcoef.alloc(2 * MAXB + 3));
+        DS_CHECK(scal.alloc(1));
         DS_CHECK(y.alloc(m));
         DS_CHECK(dsig.alloc(m + 1));
         dstate* S = dst.p;
@@ -1856,7 +1895,8 @@ private:
         // products of columns 0 .. j with u = V_j (and z = V_{j+1}), merged by k_gm_step
         auto project = [&](int j, auto lastc) {
             constexpr bool LAST = decltype(lastc)::value;
-            const int k = j + 1, nch = (k + 7) / 8, kpc = (k + nch - 1) / nch;
+            const int k = !LAST && j == 0 ? 2 : j + 1;   // step 0: (z, z) too
+            const int nch = (k + 7) / 8, kpc = (k + nch - 1) / nch;
             // 2 blocks per CU over all chunks: 15 columns of 1.72 M FP64 rows 41.1 us,
             // against 40.5 at 1, 45.3 at 4 and 43.6 at 8; 4 columns 15.9, 18.2, 18.0, 19.0;
             // 30 columns of 1.9 M FP32 rows 42.6, 50.4, 45.3, 46.2
@@ -1867,17 +1907,17 @@ private:
                 hipLaunchKernelGGL((k_gm_proj<T, C, NTB, LAST ? 1 : 2>), dim3((unsigned)gd, nch), dim3(DB), 0, st, n,
                                    k, kpc, bp, V[j], LAST ? V[j] : V[LAST ? j : j + 1], part, stop);
             });
-            hipLaunchKernelGGL((k_gm_step<LAST>), dim3(1), dim3(1024), 0, st, part, (unsigned)gd, j, Hq.p, H.p, ldh,
-                               cs.p, sn.p, g.p, dsig.p, dcoef.p, S);
+            hipLaunchKernelGGL((k_gm_step<T, LAST>), dim3(1), dim3(1024), 0, st, part, (unsigned)gd, j, Hq.p, H.p, ldh,
+                               cs.p, sn.p, g.p, dsig.p, dcoef.p, scal.p, S);
         };
         HPB_HIP(hipStreamSynchronize(st));
         HPB_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         int rc = [&]() -> int {
             DS_CHECK(apply(P.x, P.b, V[0], done));
             DS_CHECK(nrm2_async<T>(h, n, V[0], n4.p, comp, done));
-            hipLaunchKernelGGL((k_gm_start<T, double>), dim3(1), dim3(1), 0, st, S, n4.p, g.p, m, dsig.p, hist());
+            hipLaunchKernelGGL((k_gm_start<T, double>), dim3(1), dim3(1), 0, st, S, n4.p, g.p, m, dsig.p, scal.p, hist());
             for (int j = 0; j < m; ++j) {
-                DS_CHECK(apply(V[j], nullptr, V[j + 1], stop));
+                DS_CHECK(apply(V[j], nullptr, V[j + 1], stop, j == 0 ? scal.p : nullptr));
                 project(j, BF{});
                 flags([&](auto compc, auto ntc) {
                     constexpr bool C = decltype(compc)::value, NTB = decltype(ntc)::value;
@@ -1946,7 +1986,7 @@ private:
         int rc = [&]() -> int {
             DS_CHECK(apply(P.x, P.b, V[0], done));
             DS_CHECK(nrm2_async<T>(h, n, V[0], n4.p, comp, done));
-            hipLaunchKernelGGL((k_gm_start<T, T>), dim3(1), dim3(1), 0, st, S, n4.p, g.p, m, sig, hp);
+            hipLaunchKernelGGL((k_gm_start<T, T>), dim3(1), dim3(1), 0, st, S, n4.p, g.p, m, sig, (T*)nullptr, hp);
             for (int j = 0; j < m; ++j) {
                 const int k = j + 1;
                 // w = A (sig_j V_j), stored unnormalised in V[j+1]
