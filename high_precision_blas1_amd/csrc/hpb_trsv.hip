@@ -34,6 +34,7 @@
 
 #include <algorithm>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "hpb_device.hpp"
@@ -52,8 +53,8 @@ struct hpb_trsv_s {
     std::vector<int> level_ptr; // host: level l holds perm[level_ptr[l] .. level_ptr[l+1])
     int lpr = 1;
     bool all_diag = false;      // every row stores its diagonal entry
-    int4* recs = nullptr;       // device, rows by level: {row, first, end of its dependencies, diagonal entry};
-                                // null: the level kernels solve this pattern
+    int4* recs = nullptr;       // device, rows by level: {row, first dependency, their number | 256 x the lane of the
+                                // first in the level kernels, diagonal entry}; null: the level kernels solve this pattern
 };
 
 namespace hpb {
@@ -112,6 +113,13 @@ __global__ __launch_bounds__(TB) void k_trsv(int beg, int end, const int* __rest
 // that has polled FLOW_SPINS times in vain stores NaN.)  About four levels' rows are in
 // flight, so that a wave has its entries loaded when its level comes up; more pollers
 // slow the chain.
+// A plain row is summed as the LPR lanes of the level kernel sum it, entries LPR apart in
+// one sum each and the sums added in pairs, so its bits are the level kernel's: one serial
+// sum of 40 entries has 2.4 times the rounding error.  The four sums the next entries go
+// to stay in acc[0 .. 3]: acc turns by four after every four entries, and the pairs it is
+// added in are the same however far it has turned.  (One serial sum instead: 7-point
+// 128^3 681 us against 684, 150 levels of 300 rows of 24 entries 214 against 222.)  A
+// compensated row is one Dot2 sum.
 // 96 x 90 x 84 7-point (268 levels), lower / upper: 421 / 422 us, with a launch per level
 // 967 / 1083; 5-point 1000^2 (1999 levels) 2348 / 2404 (7191 / 8126); tridiagonal, 20 000
 // levels of one row, 13.4 / 14.0 ms (76.5 / 70.8).
@@ -135,12 +143,13 @@ __global__ __launch_bounds__(TB) void k_flow_init(int rows, typename flow_bits<T
     for (long i = (long)blockIdx.x * TB + threadIdx.x; i < rows; i += (long)gridDim.x * TB) w[i] = flow_bits<T>::empty;
 }
 
-template <typename T, bool COMP, bool UNIT>
+template <typename T, bool COMP, bool UNIT, int LPR>
 __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restrict__ recs, const int* __restrict__ ci,
                                                   const T* __restrict__ val, T alpha, const T* b, T* x,
                                                   typename flow_bits<T>::type* w, unsigned* next)
 {
     using U = typename flow_bits<T>::type;
+    constexpr int NA = COMP ? 1 : LPR;
     const int lane = threadIdx.x;
     for (;;) {
         unsigned chunk = 0;
@@ -150,10 +159,16 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
         if ((long)chunk * 64 >= rows) return;
         bool stored = t >= rows;
         const int4 rec = recs[stored ? rows - 1 : t];
-        const int i = rec.x, end = rec.z;
+        const int i = rec.x, end = rec.y + (rec.z & 255);
         int p = rec.y;
-        T s = alpha == T(1) ? b[i] : alpha * b[i], c = T(0);
+        const T bi = alpha == T(1) ? b[i] : alpha * b[i];
         const T d = UNIT ? T(1) : val[rec.w];
+        T acc[NA], c = T(0);
+        {
+            const int at = -(rec.z >> 8) & (NA - 1);   // lane 0's sum starts from b_i
+#pragma unroll
+            for (int k = 0; k < NA; ++k) acc[k] = k == at ? bi : T(0);
+        }
         // four entries at a time: columns, values and (once there) the solution values
         int j[4];
         T a[4], xv[4];
@@ -184,14 +199,26 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     if (p + q < end) {
-                        if (COMP) dev::dot2_step<T>(s, c, -a[q], xv[q]);
-                        else s = dev::fma_rn<T>(-a[q], xv[q], s);
+                        if (COMP) dev::dot2_step<T>(acc[0], c, -a[q], xv[q]);
+                        else acc[q % NA] = dev::fma_rn<T>(-a[q], xv[q], acc[q % NA]);
                     }
                 p += 4;
                 if (p < end) {
                     fetch();
+                    if constexpr (NA > 4) {
+                        T turned[NA];
+#pragma unroll
+                        for (int k = 0; k < NA; ++k) turned[k] = acc[(k + 4) % NA];
+#pragma unroll
+                        for (int k = 0; k < NA; ++k) acc[k] = turned[k];
+                    }
                 } else {
-                    T r = COMP ? s + c : s;
+#pragma unroll
+                    for (int m = NA / 2; m >= 1; m >>= 1)
+#pragma unroll
+                        for (int k = 0; k < NA / 2; ++k)
+                            if (k < m) acc[k] = acc[k] + acc[k + m];
+                    T r = COMP ? acc[0] + c : acc[0];
                     if (!UNIT) r = r / d;
                     U bits = __builtin_bit_cast(U, r);
                     if (bits == flow_bits<T>::empty) bits = flow_bits<T>::nan;   // this NaN means "not there"
@@ -204,8 +231,8 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
     }
 }
 
-// {row, first dependency, end, diagonal entry} of the rows in level order
-__global__ __launch_bounds__(TB) void k_flow_recs(int rows, bool upper, const int* __restrict__ perm,
+// hpb_trsv_s::recs
+__global__ __launch_bounds__(TB) void k_flow_recs(int rows, bool upper, int lpr, const int* __restrict__ perm,
                                                   const int* __restrict__ rp, const int* __restrict__ ci,
                                                   const int* __restrict__ diag, int4* __restrict__ recs)
 {
@@ -218,7 +245,7 @@ __global__ __launch_bounds__(TB) void k_flow_recs(int rows, bool upper, const in
             else hi = mid;
         }
         const int d = diag[i], after = lo + (d >= 0 ? 1 : 0);
-        recs[t] = upper ? make_int4(i, after, re, d) : make_int4(i, rb, lo, d);
+        recs[t] = upper ? make_int4(i, after, (re - after) | (after - rb) % lpr << 8, d) : make_int4(i, rb, lo - rb, d);
     }
 }
 
@@ -308,8 +335,16 @@ void trsv_all(hpb_handle_t h, const hpb_trsv_s* t, const T* val, T alpha, const 
         const long cus = h->num_cu > 0 ? h->num_cu : 256;
         const unsigned gi = (unsigned)std::max(1L, std::min(((long)t->rows + TB - 1) / TB, 4 * cus));
         hipLaunchKernelGGL((k_flow_init<T>), dim3(gi), dim3(TB), 0, st, t->rows, w, next);
-        hipLaunchKernelGGL((k_trsv_flow<T, COMP, UNIT>), dim3((unsigned)flow_waves(t->rows, nl, cus)), dim3(64), 0, st, t->rows,
-                           t->recs, t->ci, val, alpha, b, x, w, next);
+        auto go = [&](auto lprc) {
+            hipLaunchKernelGGL((k_trsv_flow<T, COMP, UNIT, decltype(lprc)::value>),
+                               dim3((unsigned)flow_waves(t->rows, nl, cus)), dim3(64), 0, st, t->rows, t->recs, t->ci,
+                               val, alpha, b, x, w, next);
+        };
+        if (COMP || t->lpr == 1) go(std::integral_constant<int, 1>{});
+        else if (t->lpr == 2) go(std::integral_constant<int, 2>{});
+        else if (t->lpr == 4) go(std::integral_constant<int, 4>{});
+        else if (t->lpr == 8) go(std::integral_constant<int, 8>{});
+        else go(std::integral_constant<int, 16>{});
         return;
     }
     for (int l = 0; l < nl; ++l) {
@@ -487,8 +522,8 @@ int hpb_csr_trsv_analysis(hpb_handle_t h, int uplo, int rows, int64_t nnz, const
             (void)hipGetLastError();
         } else {
             const unsigned g = (unsigned)std::min(((long)rows + TB - 1) / TB, 4096L);
-            hipLaunchKernelGGL(k_flow_recs, dim3(g), dim3(TB), 0, h->stream, rows, !lower, t->perm, t->rp, t->ci, t->diag,
-                               t->recs);
+            hipLaunchKernelGGL(k_flow_recs, dim3(g), dim3(TB), 0, h->stream, rows, !lower, t->lpr, t->perm, t->rp, t->ci,
+                               t->diag, t->recs);
             e = hipGetLastError();
             (void)flow_workspace(h, flow_bytes_of(rows));   // so that a captured solve finds it
         }

@@ -270,3 +270,39 @@ def test_one_launch_solves(handle, dtype):
             H.call("hpb_trsv_destroy", t)
         for v in (rp, ci, va):
             v.free()
+
+
+@pytest.mark.parametrize("deg", [1, 2, 4, 9, 17, 40, 64])
+def test_plain_rows_have_the_order_of_the_lanes(handle, deg):
+    """Plain rows in one launch: every solution entry is, bit for bit, the row's sum in the
+    order in which the lanes of the level kernels add it (the oracle's row order, the
+    entries outside the triangle set to zero), for rows of up to deg dependencies whose
+    first one lies anywhere in its row."""
+    n, r = 1500, np.random.default_rng(deg)
+    d = np.minimum(r.integers(0, 2 * deg + 1, n), deg)
+    low = np.concatenate([r.choice(i, min(i, k), replace=False) for i, k in enumerate(d)])
+    row = np.repeat(np.arange(n), np.minimum(np.arange(n), d))
+    off = np.concatenate([row * n + low, np.arange(n) * (n + 1), (n - 1 - row) * n + n - 1 - low])
+    M = sp.csr_matrix((r.uniform(-1, 1, off.size), (off // n, off % n)), shape=(n, n))
+    M.data /= max(1, deg)
+    M.setdiag(r.uniform(1, 2, n))
+    rp, ci, va, Ms = _dev_csr(handle, M)
+    mean = Ms.nnz / n
+    lpr = 1 if mean <= 1.5 else 2 if mean <= 3 else 4 if mean <= 6 else 8 if mean <= 12 else 16
+    b = r.standard_normal(n)
+    db, dx = H.DeviceArray.from_numpy(b, handle), H.DeviceArray(n, np.float64, handle)
+    for uplo in (0, 1, 2, 3):
+        say("row order", deg, lpr, uplo)
+        t = _analysis(handle, uplo, Ms, rp, ci)
+        H.call("hpb_csr_trsv_f64", handle.ptr, t, va.ptr, ctypes.c_double(1.0), db.ptr, dx.ptr, 0)
+        H.call("hpb_trsv_destroy", t)
+        x = dx.numpy()
+        at = np.repeat(np.arange(n), np.diff(Ms.indptr))
+        T = Ms.copy()
+        T.data[(Ms.indices >= at) if uplo in (0, 2) else (Ms.indices <= at)] = 0.0
+        want = O.csr_spmv(T, x, lpr=lpr, b=b)
+        if uplo in (1, 2):
+            want = want / Ms.diagonal()
+        assert want.tobytes() == x.tobytes()
+    for a in (rp, ci, va, db, dx):
+        a.free()
