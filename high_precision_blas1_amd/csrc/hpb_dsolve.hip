@@ -1256,7 +1256,7 @@ __global__ __launch_bounds__(DB) void k_ds_spmv(int rows, int tile, const int* _
 // (29.9), 16.8 M rows 116 (234).  NT: the values are loaded nontemporally, chosen when
 // the form is larger than the 256 MB MALL (16.8 M rows FP64 / FP32 229 / 116 us against
 // 247 / 144; 1.72 M rows, 113 MB of values: 24.1 against 19.1).
-template <typename T, bool CROWS, bool COMP, int MODE, int EPI, bool NT>
+template <typename T, bool CROWS, bool COMP, int MODE, int EPI, bool NT, int NC>
 __global__ __launch_bounds__(DB) void k_sd_spmv(int rows, sdia_view<T> A, const T* __restrict__ x,
                                                 const T* __restrict__ b, T* __restrict__ y, const T* __restrict__ rt,
                                                 T* __restrict__ part, const int* __restrict__ skip,
@@ -1279,7 +1279,7 @@ __global__ __launch_bounds__(DB) void k_sd_spmv(int rows, sdia_view<T> A, const 
         const long ra = in ? r : rows - 1;
         const T rtr = NQ >= 1 ? rt[ra] : T(0);
         T s = MODE == 1 ? b[ra] : T(0), c = T(0);
-        sd::row<T, CROWS, MODE == 1, NT>(A, sl, ra, x, s, c);
+        sd::row<T, CROWS, MODE == 1, NT, 0, NC>(A, sl, ra, x, s, c);
         if (in) {
             T v = CROWS ? s + c : s;
             if (alpha != T(1)) v = alpha * v;
@@ -1821,21 +1821,26 @@ private:
         long G = std::min((nsl + DB / 64 - 1) / (DB / 64), (EPI == EPI_NONE ? 16 : 6) * cus);
         G = (G + dev::XCD_COUNT - 1) / dev::XCD_COUNT * dev::XCD_COUNT;
         T* part = reinterpret_cast<T*>(h->part);
-        auto go = [&](auto crows, auto compc, auto ntc) {
+        auto go = [&](auto crows, auto compc, auto ntc, auto ncc) {
             constexpr bool CR = decltype(crows)::value, CO = decltype(compc)::value, NTB = decltype(ntc)::value;
-            hipLaunchKernelGGL((k_sd_spmv<T, CR, CO && EPI != EPI_NONE, MODE, EPI, NTB>), dim3((unsigned)G), dim3(DB), 0,
-                               h->stream, P.rows, A, x, b, y, rtv, part, skip, dalpha);
+            hipLaunchKernelGGL((k_sd_spmv<T, CR, CO && EPI != EPI_NONE, MODE, EPI, NTB, decltype(ncc)::value>),
+                               dim3((unsigned)G), dim3(DB), 0, h->stream, P.rows, A, x, b, y, rtv, part, skip, dalpha);
         };
-        auto go2 = [&](auto crows, auto compc) {
-            if (nt_mat) go(crows, compc, std::true_type{});
-            else go(crows, compc, std::false_type{});
+        auto go2 = [&](auto crows, auto compc, auto ncc) {
+            if (nt_mat) go(crows, compc, std::true_type{}, ncc);
+            else go(crows, compc, std::false_type{}, ncc);
         };
-        auto go1 = [&](auto crows) {
-            if (prm.high_precision) go2(crows, std::true_type{});
-            else go2(crows, std::false_type{});
+        auto go1 = [&](auto crows, auto ncc) {
+            if (prm.high_precision) go2(crows, std::true_type{}, ncc);
+            else go2(crows, std::false_type{}, ncc);
         };
-        if (prm.compensated_spmv) go1(std::true_type{});
-        else go1(std::false_type{});
+        // plain rows: the lanes the CSR product would take
+        const double mean = (double)P.nnz / P.rows;
+        if (prm.compensated_spmv) go1(std::true_type{}, std::integral_constant<int, 2>{});
+        else if (mean <= 8.0) go1(std::false_type{}, std::integral_constant<int, 2>{});
+        else if (mean <= 12.0) go1(std::false_type{}, std::integral_constant<int, 4>{});
+        else if (mean <= 24.0) go1(std::false_type{}, std::integral_constant<int, 8>{});
+        else go1(std::false_type{}, std::integral_constant<int, 16>{});
         return (unsigned)G;
     }
 
@@ -2364,6 +2369,18 @@ private:
     }
 
 public:
+    // one product as a solve forms it; *diagonals: K of the sliced form, 0 for CSR
+    int product(const problem<T>& pr, bool compensated, const T* x, const T* b, T* y, int* diagonals)
+    {
+        P = pr;
+        prm.compensated_spmv = compensated;
+        DS_CHECK(build_sdia());
+        if (diagonals) *diagonals = A.K;
+        if (y) DS_CHECK(apply(x, b, y, nullptr));
+        HPB_HIP(hipStreamSynchronize(P.h->stream));
+        return HPB_OK;
+    }
+
     int updates = 0;
     bool fused = false;   // BiCGStab(L): the cycle graph finishes with beta for the next cycle
 
@@ -2490,3 +2507,33 @@ template int dsolve<float>(hpb_handle_t, int, int64_t, const int*, const int*, c
                            const hpb_solver_params&, hpb_solver_result*, double*, int, dsolver_base**);
 
 }  // namespace hpb
+
+namespace {
+template <typename T>
+int product_entry(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const T* val, int compensated,
+                  const T* x, const T* b, T* y, int* diagonals)
+{
+    HPB_CLEAR_STALE();
+    HPB_REQUIRE(h && rp && ci && val && (!y || x), HPB_ERR_INVALID, "hpb_csr_solver_product: null argument");
+    HPB_REQUIRE(rows > 0 && nnz > 0, HPB_ERR_INVALID, "hpb_csr_solver_product: empty matrix");
+    hpb::dsolver<T> ds;
+    return ds.product(hpb::problem<T>{h, rows, nnz, rp, ci, val, nullptr, nullptr}, compensated != 0, x, b, y, diagonals);
+}
+}  // namespace
+
+extern "C" {
+
+int hpb_csr_solver_product_f64(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
+                               const double* val, int compensated, const double* x, const double* b, double* y,
+                               int* diagonals)
+{
+    return product_entry<double>(h, rows, nnz, row_ptr, col_ind, val, compensated, x, b, y, diagonals);
+}
+int hpb_csr_solver_product_f32(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
+                               const float* val, int compensated, const float* x, const float* b, float* y,
+                               int* diagonals)
+{
+    return product_entry<float>(h, rows, nnz, row_ptr, col_ind, val, compensated, x, b, y, diagonals);
+}
+
+}  // extern "C"

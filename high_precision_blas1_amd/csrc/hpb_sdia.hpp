@@ -12,8 +12,13 @@
 // taken when every row's columns are strictly ascending, no slice has more than
 // SD_MAXK diagonals and the K 64-row columns of all slices hold at most a quarter more
 // slots than the matrix has entries; any other matrix stays in CSR.
-// A row's entries are summed as two lanes of the CSR kernels sum them (entries 0, 2, ...
-// and 1, 3, ... apart, then merged), so up to 8 entries per row the bits are the same.
+// Where the CSR kernels take two lanes per row (a mean of more than 1.5 and up to 8
+// entries), a row's entries are summed as those lanes sum them (entries 0, 2, ... and 1,
+// 3, ... apart, then merged): the bits are the same.  Longer plain rows keep as many sums
+// as CSR has lanes, the diagonals dealt out in turn: the bits of CSR for rows that hold
+// an entry on every diagonal of their slice, no longer chains for the others.  (Two sums
+// instead: 1.1 to 1.3 times CSR's rounding error at 19 to 32 entries.)  Longer compensated
+// rows stay with two Dot2 sums.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -113,8 +118,8 @@ __global__ __launch_bounds__(SD_THREADS) void k_sdia_fill(long nsl, int rows, in
 // One row per lane: the row's product with x accumulated into (s, c), which may start
 // from a first term (b of a residual, with NEG).  sl and K are wave-uniform; lanes past
 // the last row hold no entry in any mask and pass any valid row as r.  KT > 0: A.K, known
-// to the compiler; else eight diagonals at a time.
-template <typename T, bool COMP, bool NEG, bool NT, int KT = 0>
+// to the compiler; else eight diagonals at a time.  NC: sums of a row.
+template <typename T, bool COMP, bool NEG, bool NT, int KT = 0, int NC = 2>
 __device__ __forceinline__ void row(const sdia_view<T>& A, long sl, long r, const T* __restrict__ x, T& s, T& c)
 {
     const int lane = threadIdx.x & 63;
@@ -123,6 +128,45 @@ __device__ __forceinline__ void row(const sdia_view<T>& A, long sl, long r, cons
     const int* __restrict__ off = A.off + sl * K;
     const uint64_t* __restrict__ mask = A.mask + sl * K;
     const T* __restrict__ val = A.val + sl * K * 64 + lane;
+    if constexpr (NC > 2) {
+        static_assert(!COMP && KT == 0 && (NC == 4 || NC == 8 || NC == 16), "sd::row: plain rows");
+        T acc[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) acc[k] = k == 0 ? s : T(0);
+        for (int k0 = 0; k0 < K; k0 += CH) {
+            T v[CH], xv[CH];
+            bool on[CH];
+            const int nk = K - k0;
+#pragma unroll
+            for (int k = 0; k < CH; ++k)
+                if (k < nk) {
+                    v[k] = NT ? dev::load_nt<T>(val + (long)(k0 + k) * 64) : val[(long)(k0 + k) * 64];
+                    on[k] = ((mask[k0 + k] >> lane) & 1) != 0;
+                    xv[k] = x[on[k] ? r + off[k0 + k] : r];
+                }
+#pragma unroll
+            for (int k = 0; k < CH; ++k)
+                if (k < nk) {
+                    const T t = dev::fma_rn<T>(NEG ? -v[k] : v[k], xv[k], acc[k % NC]);
+                    acc[k % NC] = on[k] ? t : acc[k % NC];
+                }
+            if (NC == 16) {   // the next eight diagonals go to the other eight sums
+#pragma unroll
+                for (int k = 0; k < CH; ++k) {
+                    const T t = acc[k];
+                    acc[k] = acc[(k + CH) % NC];
+                    acc[(k + CH) % NC] = t;
+                }
+            }
+        }
+#pragma unroll
+        for (int m = NC / 2; m >= 1; m >>= 1)
+#pragma unroll
+            for (int k = 0; k < NC / 2; ++k)
+                if (k < m) acc[k] = acc[k] + acc[k + m];
+        s = acc[0];
+        return;
+    }
     // (s, c): the sum the next entry goes to, (so, co): the other one
     T so = T(0), co = T(0);
     bool odd = false;
