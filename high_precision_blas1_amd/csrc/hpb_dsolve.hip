@@ -1553,12 +1553,15 @@ struct dbuf {
     dbuf(const dbuf&) = delete;
     dbuf& operator=(const dbuf&) = delete;
     dbuf(dbuf&& o) noexcept : p(o.p) { o.p = nullptr; }
-    ~dbuf()
+    ~dbuf() { release(); }
+    void release()
     {
         if (p) (void)hipFree(p);
+        p = nullptr;
     }
     int alloc(size_t count)
     {
+        release();
         const hipError_t e = hipMalloc((void**)&p, sizeof(T) * (count ? count : 1));
         if (e != hipSuccess) return hip_status(e, __FILE__, __LINE__, "device solver workspace");
         return HPB_OK;
@@ -1571,10 +1574,13 @@ struct graph_guard {
     graph_guard() = default;
     graph_guard(const graph_guard&) = delete;
     graph_guard& operator=(const graph_guard&) = delete;
-    ~graph_guard()
+    ~graph_guard() { release(); }
+    void release()
     {
         if (e) (void)hipGraphExecDestroy(e);
         if (g) (void)hipGraphDestroy(g);
+        e = nullptr;
+        g = nullptr;
     }
 };
 
@@ -1701,14 +1707,27 @@ public:
         hcap = hist_cap;
         reliable = rel != nullptr;
         if (rel) R = *rel;
+        DS_CHECK(plan_sdia());
+        int rc = prepare();
+        if (rc != HPB_OK && A.K > 0) {   // the form is optional: without it a solve may fit
+            A = sdia_view<T>{};
+            slab.release();
+            gg.release();
+            HPB_CLEAR_STALE();
+            rc = prepare();
+        }
+        return rc;
+    }
+    // the workspaces and the captured cycle, with the sliced-diagonal form if A.K > 0
+    int prepare()
+    {
         DS_CHECK(dst.alloc(1));
-        DS_CHECK(build_sdia());
         if (hcap) DS_CHECK(dhist.alloc(2 * (size_t)hcap));
         if (reliable) {
             DS_CHECK(r64.alloc((size_t)P.rows));
             DS_CHECK(n4d.alloc(4));
         }
-        return p.solver == HPB_SOLVER_GMRES ? setup_gmres() : setup_bicgstabl();
+        return prm.solver == HPB_SOLVER_GMRES ? setup_gmres() : setup_bicgstabl();
     }
     bool matches(const problem<T>& pr, const hpb_solver_params& p, int hist_cap) const
     {
@@ -1740,12 +1759,11 @@ private:
     dbuf<dstate> dst;
     dbuf<double> dhist;
     graph_guard gg;
-    dbuf<T> slab;                // the vectors of length rows
+    dbuf<char> slab;             // the vectors of length rows and the sliced-diagonal form
     std::vector<T*> V, U;
     T* rt = nullptr;             // shadow residual of BiCGStab(L)
     dbuf<double> H, Hq, cs, sn, g, dcoef, dsig;
-    dbuf<char> sdbuf;            // the sliced-diagonal form, when the matrix takes it
-    sdia_view<T> A{};            // A.K == 0: products run on the CSR arrays
+    sdia_view<T> A{};            // the sliced-diagonal form; A.K == 0: products run on the CSR arrays
     bool nt_mat = false;         // the form is larger than the MALL
     dbuf<T> d4, n4, coef, y, scal, da, db, gram;
     dbuf<double> r64, n4d;
@@ -1753,56 +1771,62 @@ private:
 
     double* hist() { return hcap ? dhist.p : nullptr; }
 
-    // nv + nu vectors of n in one allocation (31 allocations of 14 MB took 8 ms with their
-    // releases, one of 430 MB 0.3 ms), every one 256-byte aligned; U ends with r~.
+    // nv + nu vectors of n, every one 256-byte aligned, and the sliced-diagonal form when
+    // plan_sdia found one, in one allocation (31 allocations of 14 MB took 8 ms with their
+    // releases, one of 430 MB 0.3 ms); U ends with r~.
     int alloc_vectors(size_t n, int nv, int nu)
     {
         const size_t per = 256 / sizeof(T), stride = (n + per - 1) / per * per;
-        DS_CHECK(slab.alloc(stride * (size_t)(nv + nu)));
+        const size_t vecs = sizeof(T) * stride * (size_t)(nv + nu);
+        DS_CHECK(slab.alloc(vecs + form_bytes()));
+        T* const v = reinterpret_cast<T*>(slab.p);
         V.resize(nv);
         U.resize(nu);
-        for (int j = 0; j < nv; ++j) V[j] = slab.p + stride * (size_t)j;
-        for (int j = 0; j < nu; ++j) U[j] = slab.p + stride * (size_t)(nv + j);
+        for (int j = 0; j < nv; ++j) V[j] = v + stride * (size_t)j;
+        for (int j = 0; j < nu; ++j) U[j] = v + stride * (size_t)(nv + j);
         rt = nu > 0 ? U[nu - 1] : nullptr;
-        return HPB_OK;
+        return A.K > 0 ? fill_sdia(slab.p + vecs) : HPB_OK;
     }
 
-    // The sliced-diagonal form of the matrix (hpb_sdia.hpp), when it fits and the system
-    // has at least 32768 rows: below, a product is bound by its launch (10560 rows: 3.1
-    // against 3.3 us) and the two passes and the copy back would not pay.  A form that
-    // cannot be allocated leaves the products on CSR.
-    int build_sdia()
+    // Decides on the sliced-diagonal form of the matrix (hpb_sdia.hpp): A.K > 0 when it
+    // fits and the system has at least 32768 rows: below, a product is bound by its launch
+    // (10560 rows: 3.1 against 3.3 us) and the two passes and the copy back would not pay.
+    int plan_sdia()
     {
         hpb_handle_t h = P.h;
         hipStream_t st = h->stream;
         A = sdia_view<T>{};
         if (P.rows < 32768 || P.nnz > (int64_t)SD_MAXK * P.rows) return HPB_OK;
-        const long nsl = ((long)P.rows + 63) / 64;
-        const size_t cus = (size_t)(h->num_cu > 0 ? h->num_cu : 256);
-        const unsigned G = (unsigned)std::min<size_t>((size_t)(nsl + 3) / 4, 8 * cus);
         int* info = reinterpret_cast<int*>(h->dres);
         hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(DB), 0, st, (size_t)2, info, 0);
-        hipLaunchKernelGGL(sd::k_sdia_count, dim3(G), dim3(SD_THREADS), 0, st, nsl, P.rows, P.rp, P.ci, info);
+        hipLaunchKernelGGL(sd::k_sdia_count, dim3(sdia_grid()), dim3(SD_THREADS), 0, st, slices(), P.rows, P.rp, P.ci, info);
         HPB_LAUNCH_CHECK();
         HPB_HIP(hipMemcpyAsync(h->hres, info, 2 * sizeof(int), hipMemcpyDeviceToHost, st));
         HPB_HIP(hipStreamSynchronize(st));
         const int K = reinterpret_cast<const int*>(h->hres)[0], bad = reinterpret_cast<const int*>(h->hres)[1];
-        const int64_t slots = (int64_t)nsl * 64 * K;
-        if (bad || K < 1 || 4 * slots > 5 * P.nnz + 1024) return HPB_OK;
-        const size_t bv = sizeof(T) * (size_t)slots, bm = sizeof(uint64_t) * (size_t)nsl * K;
-        const size_t bytes = bv + bm + sizeof(int) * (size_t)nsl * K;
-        if (hipMalloc((void**)&sdbuf.p, bytes) != hipSuccess) {
-            sdbuf.p = nullptr;
-            (void)hipGetLastError();
-            return HPB_OK;
-        }
-        A.K = K;
-        A.val = reinterpret_cast<const T*>(sdbuf.p);
-        A.mask = reinterpret_cast<const uint64_t*>(sdbuf.p + bv);
-        A.off = reinterpret_cast<const int*>(sdbuf.p + bv + bm);
-        nt_mat = bytes > (size_t)256 * 1024 * 1024;
-        hipLaunchKernelGGL((sd::k_sdia_fill<T>), dim3(G), dim3(SD_THREADS), 0, st, nsl, P.rows, K, P.rp, P.ci, P.val,
-                           const_cast<int*>(A.off), const_cast<uint64_t*>(A.mask), const_cast<T*>(A.val));
+        if (!bad && K >= 1 && 4 * (int64_t)slices() * 64 * K <= 5 * P.nnz + 1024) A.K = K;
+        return HPB_OK;
+    }
+
+    long slices() const { return ((long)P.rows + 63) / 64; }
+    size_t form_slots() const { return (size_t)slices() * (size_t)A.K; }
+    size_t form_bytes() const { return form_slots() * (64 * sizeof(T) + sizeof(uint64_t) + sizeof(int)); }
+    unsigned sdia_grid() const
+    {
+        const long cus = P.h->num_cu > 0 ? P.h->num_cu : 256;
+        return (unsigned)std::min((slices() + 3) / 4, 8 * cus);
+    }
+
+    int fill_sdia(char* at)
+    {
+        const size_t bv = 64 * sizeof(T) * form_slots(), bm = sizeof(uint64_t) * form_slots();
+        A.val = reinterpret_cast<const T*>(at);
+        A.mask = reinterpret_cast<const uint64_t*>(at + bv);
+        A.off = reinterpret_cast<const int*>(at + bv + bm);
+        nt_mat = form_bytes() > (size_t)256 * 1024 * 1024;
+        hipLaunchKernelGGL((sd::k_sdia_fill<T>), dim3(sdia_grid()), dim3(SD_THREADS), 0, P.h->stream, slices(), P.rows, A.K,
+                           P.rp, P.ci, P.val, const_cast<int*>(A.off), const_cast<uint64_t*>(A.mask),
+                           const_cast<T*>(A.val));
         HPB_LAUNCH_CHECK();
         return HPB_OK;
     }
@@ -2374,7 +2398,8 @@ public:
     {
         P = pr;
         prm.compensated_spmv = compensated;
-        DS_CHECK(build_sdia());
+        DS_CHECK(plan_sdia());
+        DS_CHECK(alloc_vectors(0, 0, 0));
         if (diagonals) *diagonals = A.K;
         if (y) DS_CHECK(apply(x, b, y, nullptr));
         HPB_HIP(hipStreamSynchronize(P.h->stream));
