@@ -726,7 +726,7 @@ __global__ __launch_bounds__(256) void k_bslices(int ntiles, const btile* __rest
                     mask[sl * BDIAG + e] = m;
                 }
             };
-            const int n = sd::walk_slice(r0, t.r1, rp, col, put);
+            const int n = sd::walk_slice(r0, t.r1, rp, [&](int p) { return col[p]; }, put);
             for (int e = n < 0 ? 0 : n; e < BDIAG; ++e) put(e, 0, 0, -1);
         }
     }

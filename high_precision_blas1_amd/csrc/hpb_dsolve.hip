@@ -1696,14 +1696,18 @@ class dsolver : public dsolver_base {
 public:
     problem<T> P{};
     hpb_solver_params prm{};
+    double target = 0.0;
     int hcap = 0;
     bool reliable = false;
     rel64 R{};
 
-    int setup(const problem<T>& pr, const hpb_solver_params& p, int hist_cap, const rel64* rel = nullptr)
+    // target_tol: the relative tolerance of all the runs together
+    int setup(const problem<T>& pr, const hpb_solver_params& p, int hist_cap, double target_tol,
+              const rel64* rel = nullptr)
     {
         P = pr;
         prm = p;
+        target = target_tol;
         hcap = hist_cap;
         reliable = rel != nullptr;
         if (rel) R = *rel;
@@ -1788,15 +1792,33 @@ private:
         return A.K > 0 ? fill_sdia(slab.p + vecs) : HPB_OK;
     }
 
+    // Whether the sliced-diagonal form is worth its two passes, a copy back and its memory
+    // (60 us at 100 k rows of 7 entries, 0.1 ms at 1 M, 0.3 ms at 1 M of 27, and up to 0.6
+    // ms more where the allocation leaves the runtime's cache).  Smaller products are bound
+    // by their launch in either form, and a solve to a loose tolerance may end after a few:
+    // four products per digit are counted on.  Whole solves on rows of 5 to 32 diagonals,
+    // sliced against CSR, BiCGStab(2):
+    //   to 1e-10, plain: 33 k rows -3 to +7 %, 50 k -12 to -3, 100 k -20 to -4, 1 M -48 to -11;
+    //   compensated: 33 k -3 to +18 %, 70 k -11 to +3, 100 k -14 to +2 (7 diagonals), 150 k
+    //     -18 to -5;
+    //   to 1e-3, plain: 50 k -2 to +5 %, 70 k -6 to +4, 100 k -10 to 0, 1 M -34 to +1;
+    //   to 1e-1: -1 to +14 % at 100 k, -21 to +32 at 1 M.
+    bool form_pays() const
+    {
+        const double each = prm.solver == HPB_SOLVER_GMRES ? 1.0 : 2.0;   // products per iteration
+        const double products = std::min(-4.0 * std::log10(std::max(target, 1e-16)), each * prm.max_iters);
+        const double weight = prm.compensated_spmv ? 0.5 : 1.0;
+        return products >= 12.0 && weight * P.rows >= 49152.0 && weight * P.rows * products >= 1.2e6;
+    }
+
     // Decides on the sliced-diagonal form of the matrix (hpb_sdia.hpp): A.K > 0 when it
-    // fits and the system has at least 32768 rows: below, a product is bound by its launch
-    // (10560 rows: 3.1 against 3.3 us) and the two passes and the copy back would not pay.
+    // fits and pays.
     int plan_sdia()
     {
         hpb_handle_t h = P.h;
         hipStream_t st = h->stream;
         A = sdia_view<T>{};
-        if (P.rows < 32768 || P.nnz > (int64_t)SD_MAXK * P.rows) return HPB_OK;
+        if (!form_pays() || P.nnz > (int64_t)SD_MAXK * P.rows) return HPB_OK;
         int* info = reinterpret_cast<int*>(h->dres);
         hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(DB), 0, st, (size_t)2, info, 0);
         hipLaunchKernelGGL(sd::k_sdia_count, dim3(sdia_grid()), dim3(SD_THREADS), 0, st, slices(), P.rows, P.rp, P.ci, info);
@@ -1824,9 +1846,11 @@ private:
         A.mask = reinterpret_cast<const uint64_t*>(at + bv);
         A.off = reinterpret_cast<const int*>(at + bv + bm);
         nt_mat = form_bytes() > (size_t)256 * 1024 * 1024;
-        hipLaunchKernelGGL((sd::k_sdia_fill<T>), dim3(sdia_grid()), dim3(SD_THREADS), 0, P.h->stream, slices(), P.rows, A.K,
-                           P.rp, P.ci, P.val, const_cast<int*>(A.off), const_cast<uint64_t*>(A.mask),
-                           const_cast<T*>(A.val));
+        const long cus = P.h->num_cu > 0 ? P.h->num_cu : 256;
+        const unsigned lds = (unsigned)((sizeof(T) + sizeof(int)) * 64 * (size_t)A.K);
+        hipLaunchKernelGGL((sd::k_sdia_fill<T>), dim3((unsigned)std::min(slices(), 32 * cus)), dim3(64), lds, P.h->stream,
+                           slices(), P.rows, A.K, P.rp, P.ci, P.val, const_cast<int*>(A.off),
+                           const_cast<uint64_t*>(A.mask), const_cast<T*>(A.val));
         HPB_LAUNCH_CHECK();
         return HPB_OK;
     }
@@ -2394,10 +2418,11 @@ private:
 
 public:
     // one product as a solve forms it; *diagonals: K of the sliced form, 0 for CSR
-    int product(const problem<T>& pr, bool compensated, const T* x, const T* b, T* y, int* diagonals)
+    int product(const problem<T>& pr, const hpb_solver_params& p, const T* x, const T* b, T* y, int* diagonals)
     {
         P = pr;
-        prm.compensated_spmv = compensated;
+        prm = p;
+        target = p.rel_tol;
         DS_CHECK(plan_sdia());
         DS_CHECK(alloc_vectors(0, 0, 0));
         if (diagonals) *diagonals = A.K;
@@ -2427,11 +2452,12 @@ public:
 // (iters, converged, breakdown, resid_norm, rhs_norm, history_len) and history.
 // cache (optional): a solver object kept by the caller between calls with the
 // same operands; *cache is replaced when the operands or parameters change and
-// must be released with dsolve_release.
+// must be released with dsolve_release.  target_tol: with a cache, the relative tolerance
+// the solves reach together.
 template <typename T>
 int dsolve(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const T* val, const T* b, T* x,
            const hpb_solver_params& p, hpb_solver_result* res, double* history, int history_cap,
-           dsolver_base** cache)
+           dsolver_base** cache, double target_tol)
 {
     HPB_REQUIRE(p.solver != HPB_SOLVER_GMRES || (p.restart >= 1 && p.restart < MAXB), HPB_ERR_INVALID,
                 "device solver: GMRES restart must be in [1, 255]");
@@ -2451,7 +2477,7 @@ int dsolve(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, 
     }
     if (!ds) {
         ds = cache ? new dsolver<T>() : &local;
-        const int rc = ds->setup(P, p, hcap);
+        const int rc = ds->setup(P, p, hcap, cache ? target_tol : p.rel_tol);
         if (rc != HPB_OK) {
             if (cache) delete ds;
             return rc;
@@ -2494,7 +2520,7 @@ int dsolve_reliable(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const 
     p.rel_tol = rel_tol;   // the monitor tests the FP64 true residual against the final tolerance
     rel64 R{val64, b64, x64, delta, mscale};
     dsolver<float> ds;
-    DS_CHECK(ds.setup(P, p, 0, &R));
+    DS_CHECK(ds.setup(P, p, 0, rel_tol, &R));
     dstate out{};
     DS_CHECK(ds.run(p, &out));
     res->iters = out.iters;
@@ -2527,38 +2553,38 @@ int absmax_pow2_scale(hpb_handle_t h, size_t n, const double* x, double* scale)
 }
 
 template int dsolve<double>(hpb_handle_t, int, int64_t, const int*, const int*, const double*, const double*,
-                            double*, const hpb_solver_params&, hpb_solver_result*, double*, int, dsolver_base**);
+                            double*, const hpb_solver_params&, hpb_solver_result*, double*, int, dsolver_base**, double);
 template int dsolve<float>(hpb_handle_t, int, int64_t, const int*, const int*, const float*, const float*, float*,
-                           const hpb_solver_params&, hpb_solver_result*, double*, int, dsolver_base**);
+                           const hpb_solver_params&, hpb_solver_result*, double*, int, dsolver_base**, double);
 
 }  // namespace hpb
 
 namespace {
 template <typename T>
-int product_entry(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const T* val, int compensated,
-                  const T* x, const T* b, T* y, int* diagonals)
+int product_entry(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const T* val,
+                  const hpb_solver_params* p, const T* x, const T* b, T* y, int* diagonals)
 {
     HPB_CLEAR_STALE();
-    HPB_REQUIRE(h && rp && ci && val && (!y || x), HPB_ERR_INVALID, "hpb_csr_solver_product: null argument");
+    HPB_REQUIRE(h && rp && ci && val && p && (!y || x), HPB_ERR_INVALID, "hpb_csr_solver_product: null argument");
     HPB_REQUIRE(rows > 0 && nnz > 0, HPB_ERR_INVALID, "hpb_csr_solver_product: empty matrix");
     hpb::dsolver<T> ds;
-    return ds.product(hpb::problem<T>{h, rows, nnz, rp, ci, val, nullptr, nullptr}, compensated != 0, x, b, y, diagonals);
+    return ds.product(hpb::problem<T>{h, rows, nnz, rp, ci, val, nullptr, nullptr}, *p, x, b, y, diagonals);
 }
 }  // namespace
 
 extern "C" {
 
 int hpb_csr_solver_product_f64(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
-                               const double* val, int compensated, const double* x, const double* b, double* y,
-                               int* diagonals)
+                               const double* val, const hpb_solver_params* p, const double* x, const double* b,
+                               double* y, int* diagonals)
 {
-    return product_entry<double>(h, rows, nnz, row_ptr, col_ind, val, compensated, x, b, y, diagonals);
+    return product_entry<double>(h, rows, nnz, row_ptr, col_ind, val, p, x, b, y, diagonals);
 }
 int hpb_csr_solver_product_f32(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
-                               const float* val, int compensated, const float* x, const float* b, float* y,
+                               const float* val, const hpb_solver_params* p, const float* x, const float* b, float* y,
                                int* diagonals)
 {
-    return product_entry<float>(h, rows, nnz, row_ptr, col_ind, val, compensated, x, b, y, diagonals);
+    return product_entry<float>(h, rows, nnz, row_ptr, col_ind, val, p, x, b, y, diagonals);
 }
 
 }  // extern "C"

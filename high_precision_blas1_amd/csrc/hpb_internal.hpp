@@ -101,7 +101,7 @@ struct dsolver_base {
 template <typename T>
 int dsolve(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const T* val, const T* b, T* x,
            const hpb_solver_params& p, hpb_solver_result* res, double* history, int history_cap,
-           dsolver_base** cache = nullptr);
+           dsolver_base** cache = nullptr, double target_tol = 0.0);
 void dsolve_release(dsolver_base* cache);
 // FP32 BiCGStab(L) iterations with reliable updates of an FP64 solution
 int dsolve_reliable(hpb_handle_t h, int rows, int64_t nnz, const int* rp, const int* ci, const float* val32,

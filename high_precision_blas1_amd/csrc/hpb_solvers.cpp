@@ -336,7 +336,7 @@ int hpb_csr_solve_ir_f64(hpb_handle_t h, int rows, int64_t nnz, const int* row_p
             hpb_solver_result ir{};
             if (use_device(*inner)) {
                 const int rc = hpb::dsolve<float>(h, rows, nnz, row_ptr, col_ind, val32, r32, d32, *inner, &ir,
-                                                  nullptr, 0, &inner_cache.c);
+                                                  nullptr, 0, &inner_cache.c, rel_tol);
                 if (rc != HPB_OK) return rc;
             } else if (inner->preconditioner == HPB_PRECOND_ILU0) {
                 if (!ilu32) {

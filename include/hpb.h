@@ -449,16 +449,16 @@ void hpb_solver_params_default(hpb_solver_params* p);
 int hpb_csr_solve_f64(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
                       const double* val, const double* b, double* x, const hpb_solver_params* p,
                       hpb_solver_result* res, double* history, int history_cap);
-/* One product y = A x, or y = b - A x with b, as the device-resident solvers form it
- * (y null: none): the matrix is first rewritten into slices of diagonals where a solve
- * would do so.  *diagonals (optional): the diagonals per slice, 0 when the product runs
- * on the CSR arrays.  For checks of a matrix's form and rounding; it allocates and frees
- * the rewritten matrix on each call. */
+/* One product y = A x, or y = b - A x with b, as a device-resident solve with the
+ * parameters p forms it (y null: none): the matrix is first rewritten into slices of
+ * diagonals where that solve would do so.  *diagonals (optional): the diagonals per slice,
+ * 0 when the product runs on the CSR arrays.  For checks of a matrix's form and rounding;
+ * it allocates and frees the rewritten matrix on each call. */
 int hpb_csr_solver_product_f64(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
-                               const double* val, int compensated, const double* x, const double* b, double* y,
-                               int* diagonals);
+                               const double* val, const hpb_solver_params* p, const double* x, const double* b,
+                               double* y, int* diagonals);
 int hpb_csr_solver_product_f32(hpb_handle_t h, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
-                               const float* val, int compensated, const float* x, const float* b, float* y,
+                               const float* val, const hpb_solver_params* p, const float* x, const float* b, float* y,
                                int* diagonals);
 /* Mixed precision (new): FP32 copies of the values and FP32 Krylov vectors with
  * compensated FP32 dots inside, FP64 iterative refinement outside:
