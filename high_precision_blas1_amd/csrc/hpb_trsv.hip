@@ -299,6 +299,28 @@ long flow_waves(int rows, int nlev, long cus)
     return std::max(8L, std::min(cus, (4 * width + 63) / 64));
 }
 
+// Whether one launch for all levels beats a launch per level.  It saves about 2 us a level,
+// but one lane walks each row, 64 rows to a wave, and the waves at work are few: long rows
+// cost a start of their own, wide levels fill the device better in a launch each.  Lower
+// solves of levels of equal width, plain, one launch / a launch per level, us:
+//   2 dependencies: 4 levels of 100 rows 8 / 11, of 6000 14 / 12; 12 of 6000 25 / 33;
+//     150 of 15 000 436 / 557, of 22 000 632 / 563;
+//   12: 6 levels of 1000 16 / 18, of 6000 23 / 18; 50 of 11 000 150 / 178, of 15 000 197 / 196;
+//   24: 14 levels of 300 35 / 40, of 3000 45 / 42; 26 of 3000 64 / 89; 50 of 11 000 220 / 227;
+//   48: 26 levels of 300 78 / 79 (compensated 89 / 84); 50 of 300 134 / 154, of 8000 280 / 268;
+//   60: 12 levels of 1000 56 / 40, 40 of 1000 137 / 178.
+// 7-point grids, 256^3 (766 levels, 21.9 k rows on average) 3507 / 4278; 100 000 random rows
+// of 2.6 dependencies, the longest of 20, in 26 levels 39 / 85.
+bool flow_pays(int rows, int nlev, int longest, int64_t deps)
+{
+    const double width = (double)rows / nlev, per_level = (double)deps / nlev;
+    const double length = std::max((double)deps / rows, 0.5 * longest);
+    if (longest > 64 || per_level > 250000.0) return false;
+    if (width <= 1024.0) return nlev >= std::max(4.0, 0.6 * length);
+    if (width > (nlev < 24 ? 8192.0 : nlev < 100 ? 11264.0 : nlev < 500 ? 16384.0 : 24576.0)) return false;
+    return nlev >= (length <= 4.0 ? 6.0 : std::max(12.0, 0.75 * length));
+}
+
 // The handle's workspace of one-launch solves, at least `bytes`; null when it cannot be
 // had (no memory, or the stream is being captured and it would have to grow).  A buffer
 // that is outgrown stays allocated until the handle goes: a captured solve may use it.
@@ -505,12 +527,14 @@ int hpb_csr_trsv_analysis(hpb_handle_t h, int uplo, int rows, int64_t nnz, const
     t->all_diag = std::all_of(diag.begin(), diag.end(), [](int d) { return d >= 0; });
     const double mean = (double)nnz / rows;
     t->lpr = mean <= 1.5 ? 1 : mean <= 3.0 ? 2 : mean <= 6.0 ? 4 : mean <= 12.0 ? 8 : 16;
-    // one launch for all levels: rows of up to 64 dependencies (one lane forms a row),
-    // at least four levels, of 32768 rows on average at most (wider ones fill the device
-    // in a launch of their own: 1 M random rows in 12 levels 86 us that way)
     int longest = 0;
-    for (int i = 0; i < rows; ++i) longest = std::max(longest, lower ? lend[i] - rp[i] : rp[i + 1] - lend[i]);
-    const bool flow = longest <= 64 && nlev >= 4 && (int64_t)rows <= (int64_t)nlev * 32768;
+    int64_t deps = 0;
+    for (int i = 0; i < rows; ++i) {
+        const int d = lower ? lend[i] - rp[i] : rp[i + 1] - lend[i];   // an upper row's diagonal counts
+        longest = std::max(longest, d);
+        deps += d;
+    }
+    const bool flow = flow_pays(rows, nlev, longest, deps);
     hipError_t e = hipMalloc((void**)&t->perm, sizeof(int) * rows);
     if (e == hipSuccess) e = hipMalloc((void**)&t->diag, sizeof(int) * rows);
     if (e == hipSuccess) e = hipMemcpyAsync(t->perm, perm.data(), sizeof(int) * rows, hipMemcpyHostToDevice, h->stream);
@@ -544,6 +568,13 @@ int hpb_csr_trsv_levels(hpb_trsv_t t, int* nlevels)
 {
     HPB_REQUIRE(t && nlevels, HPB_ERR_INVALID, "hpb_csr_trsv_levels: null argument");
     *nlevels = (int)t->level_ptr.size() - 1;
+    return HPB_OK;
+}
+
+int hpb_csr_trsv_launches(hpb_trsv_t t, int* launches)
+{
+    HPB_REQUIRE(t && launches, HPB_ERR_INVALID, "hpb_csr_trsv_launches: null argument");
+    *launches = t->recs ? 2 : (int)t->level_ptr.size() - 1;
     return HPB_OK;
 }
 

@@ -374,6 +374,8 @@ typedef struct hpb_trsv_s* hpb_trsv_t;
 int hpb_csr_trsv_analysis(hpb_handle_t h, int uplo, int rows, int64_t nnz, const int* row_ptr, const int* col_ind,
                           hpb_trsv_t* out);
 int hpb_csr_trsv_levels(hpb_trsv_t t, int* nlevels);
+/* kernel launches of a solve: 2 (its workspace and all levels), or one per level */
+int hpb_csr_trsv_launches(hpb_trsv_t t, int* launches);
 int hpb_trsv_destroy(hpb_trsv_t t);
 int hpb_csr_trsv_f64(hpb_handle_t h, hpb_trsv_t t, const double* val, double alpha, const double* b, double* x,
                      int compensated);

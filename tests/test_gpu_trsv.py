@@ -241,6 +241,11 @@ def test_one_launch_solves(handle, dtype):
         for uplo in (0, 1, 2, 3):
             say("one launch", suf, name, uplo)
             t = _analysis(handle, uplo, Ms, rp, ci)
+            levels, launches = ctypes.c_int(), ctypes.c_int()
+            H.call("hpb_csr_trsv_levels", t, ctypes.byref(levels))
+            H.call("hpb_csr_trsv_launches", t, ctypes.byref(launches))
+            one = levels.value >= 4 and name != "long row"   # (its upper triangle is the diagonal)
+            assert launches.value == (2 if one else levels.value), (name, uplo)
             lower, unit = uplo in (0, 2), uplo in (0, 3)
             T = (sp.tril(Md, -1) if lower else sp.triu(Md, 1)) + (sp.identity(n) if unit else sp.diags(Md.diagonal()))
             ref = spla.spsolve_triangular(T.tocsr(), b.astype(np.float64), lower=lower)
@@ -305,4 +310,32 @@ def test_plain_rows_have_the_order_of_the_lanes(handle, deg):
             want = want / Ms.diagonal()
         assert want.tobytes() == x.tobytes()
     for a in (rp, ci, va, db, dx):
+        a.free()
+
+
+@pytest.mark.parametrize("deps,nlev,width,one", [
+    (2, 3, 100, False), (2, 4, 100, True), (2, 5, 6000, False), (2, 6, 6000, True), (2, 23, 9000, False),
+    (2, 24, 9000, True), (2, 24, 12000, False), (12, 5, 100, False), (12, 6, 100, True), (12, 11, 3000, False),
+    (12, 12, 3000, True), (24, 16, 3000, False), (24, 17, 3000, True), (60, 34, 300, False), (60, 35, 300, True),
+    (48, 40, 6000, False), (66, 80, 70, False)])
+def test_where_one_launch_is_taken(handle, deps, nlev, width, one):
+    """Rows of the given dependencies in levels of equal width: one launch only where it
+    was measured faster than a launch per level."""
+    say("launches", deps, nlev, width)
+    n = nlev * width
+    i = np.arange(width, n)
+    lev = i // width
+    # deps rows of the level before, evenly spaced from the row's own place on
+    col = ((lev - 1) * width)[:, None] + (i[:, None] + (np.arange(deps) * (width // deps))[None]) % width
+    rowl = np.repeat(i, deps)
+    M = (sp.csr_matrix((np.ones(rowl.size), (rowl, col.ravel())), shape=(n, n)) + sp.identity(n)).tocsr()
+    rp, ci, va, Ms = _dev_csr(handle, M)
+    t = _analysis(handle, 0, Ms, rp, ci)
+    levels, launches = ctypes.c_int(), ctypes.c_int()
+    H.call("hpb_csr_trsv_levels", t, ctypes.byref(levels))
+    H.call("hpb_csr_trsv_launches", t, ctypes.byref(launches))
+    H.call("hpb_trsv_destroy", t)
+    assert levels.value == nlev
+    assert launches.value == (2 if one else nlev)
+    for a in (rp, ci, va):
         a.free()
