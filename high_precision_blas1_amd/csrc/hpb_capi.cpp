@@ -36,7 +36,7 @@ int wait_host_result(hpb_handle_t h, unsigned long long seq)
     const auto t0 = std::chrono::steady_clock::now();
     for (;;) {
         for (int i = 0; i < 64; ++i) {
-            if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == seq) return HPB_OK;
+            if (__atomic_load_n(p, __ATOMIC_ACQUIRE) == seq) return flow_status(h);
             __builtin_ia32_pause();
         }
         if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(1)) break;
@@ -44,7 +44,17 @@ int wait_host_result(hpb_handle_t h, unsigned long long seq)
     HPB_HIP(hipStreamSynchronize(h->stream));
     HPB_REQUIRE(__atomic_load_n(p, __ATOMIC_ACQUIRE) == seq, HPB_ERR_UNSUPPORTED,
                 "blocking call: the stream is idle and the result was not published");
-    return HPB_OK;
+    return flow_status(h);
+}
+
+int flow_status(hpb_handle_t h)
+{
+    int* const p = &host_flag_of(h)->flow_gave_up;
+    if (__atomic_load_n(p, __ATOMIC_RELAXED) == 0) return HPB_OK;
+    __atomic_store_n(p, 0, __ATOMIC_RELAXED);
+    set_error(__FILE__, __LINE__,
+              "hpb_csr_trsv: a one-launch solve waited for a value in vain and stored NaN (hpb_set_trsv_wait_limit)");
+    return HPB_ERR_UNSUPPORTED;
 }
 
 }  // namespace hpb
@@ -154,6 +164,13 @@ int hpb_synchronize(hpb_handle_t h)
 {
     HPB_REQUIRE(h, HPB_ERR_INVALID, "hpb_synchronize: null handle");
     HPB_HIP(hipStreamSynchronize(h->stream));
+    return hpb::flow_status(h);
+}
+
+int hpb_set_trsv_wait_limit(hpb_handle_t h, uint32_t polls)
+{
+    HPB_REQUIRE(h, HPB_ERR_INVALID, "hpb_set_trsv_wait_limit: null handle");
+    h->flow_spins = polls;
     return HPB_OK;
 }
 
@@ -195,7 +212,7 @@ int hpb_memcpy_d2h(hpb_handle_t h, void* dst, const void* src, size_t bytes)
     if (bytes == 0) return HPB_OK;
     HPB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, h->stream));
     HPB_HIP(hipStreamSynchronize(h->stream));
-    return HPB_OK;
+    return hpb::flow_status(h);
 }
 
 int hpb_memcpy_d2d(hpb_handle_t h, void* dst, const void* src, size_t bytes)

@@ -35,6 +35,7 @@ struct hpb_handle_s {
     size_t hstage_bytes = 0;
     std::vector<void*> flow;        // device workspaces of the one-launch triangular solves, the last in use
     size_t flow_bytes = 0;          // ... and its size
+    unsigned flow_spins = 1u << 22; // ... and the bound of a row's polls in vain (hpb_set_trsv_wait_limit)
     hipEvent_t ev[2] = {nullptr, nullptr};
     hpb_tuning_t tune_red[2];       // two-input reductions (dot), [0] f64, [1] f32
     hpb_tuning_t tune_red1[2];      // one-input reductions (sum, asum, nrm2)
@@ -65,6 +66,7 @@ struct nrm_fix {
 struct host_flag {
     unsigned long long seq;
     int need;
+    int flow_gave_up;   // a one-launch triangular solve gave up a wait (k_trsv_flow); taken by flow_status
 };
 inline host_flag* host_flag_of(const hpb_handle_s* h)
 {
@@ -72,6 +74,8 @@ inline host_flag* host_flag_of(const hpb_handle_s* h)
 }
 // waits until call `seq` has published its results in hres
 int wait_host_result(hpb_handle_t h, unsigned long long seq);
+// error status, once, when a triangular solve that has finished gave up a wait
+int flow_status(hpb_handle_t h);
 
 void set_error(const char* file, int line, const std::string& msg);
 // looks up the current device's address of the no-allocation scratch array

@@ -109,8 +109,11 @@ __global__ __launch_bounds__(TB) void k_trsv(int beg, int end, const int* __rest
 // only depend on earlier levels, so on earlier positions of the chunk order: the wave
 // that holds the smallest unfinished chunk never waits for a chunk nobody has taken, and
 // every wait ends whatever waves are resident; a row of the same wave is stored inside
-// the polling loop, whose exit is uniform.  (The polls are bounded all the same: a wave
-// that has polled FLOW_SPINS times in vain stores NaN.)  About four levels' rows are in
+// the polling loop, whose exit is uniform.  (The polls are bounded all the same: after
+// hpb_handle_s::flow_spins polls for its chunk a wave takes NaN for the values that are
+// missing and marks the handle's host record, which its next call that waits reports.  The
+// longest legal wait, 256 chunks of 64 levels in turn, is some 20 ms, the bound seconds.)
+// About four levels' rows are in
 // flight, so that a wave has its entries loaded when its level comes up; more pollers
 // slow the chain.
 // A plain row is summed as the LPR lanes of the level kernel sum it, entries LPR apart in
@@ -132,7 +135,6 @@ template <> struct flow_bits<float> {
     using type = unsigned;
     static constexpr type empty = 0xffc5a30fu, nan = 0x7fc00000u;
 };
-constexpr unsigned FLOW_SPINS = 1u << 22;
 
 // w := FLOW_EMPTY, *next := 0
 template <typename T>
@@ -146,7 +148,8 @@ __global__ __launch_bounds__(TB) void k_flow_init(int rows, typename flow_bits<T
 template <typename T, bool COMP, bool UNIT, int LPR>
 __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restrict__ recs, const int* __restrict__ ci,
                                                   const T* __restrict__ val, T alpha, const T* b, T* x,
-                                                  typename flow_bits<T>::type* w, unsigned* next)
+                                                  typename flow_bits<T>::type* w, unsigned* next, unsigned spins,
+                                                  int* gave_up)
 {
     using U = typename flow_bits<T>::type;
     constexpr int NA = COMP ? 1 : LPR;
@@ -184,6 +187,7 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
             }
         };
         if (!stored) fetch();
+        // spin: uniform, and never reset (counts per lane or since the last row cost 1 to 2 %)
         for (unsigned spin = 0; __ballot(!stored) != 0; ++spin) {
             if (stored) continue;
             U v[4];
@@ -191,7 +195,7 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
             for (int q = 0; q < 4; ++q) v[q] = __hip_atomic_load(w + j[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                if (((wait >> q) & 1u) && (v[q] != flow_bits<T>::empty || spin >= FLOW_SPINS)) {
+                if (((wait >> q) & 1u) && (v[q] != flow_bits<T>::empty || spin >= spins)) {
                     xv[q] = __builtin_bit_cast(T, v[q]);
                     wait &= ~(1u << q);
                 }
@@ -224,6 +228,7 @@ __global__ __launch_bounds__(64) void k_trsv_flow(int rows, const int4* __restri
                     if (bits == flow_bits<T>::empty) bits = flow_bits<T>::nan;   // this NaN means "not there"
                     __hip_atomic_store(w + i, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     x[i] = r;
+                    if (spin >= spins) __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                     stored = true;
                 }
             }
@@ -360,7 +365,7 @@ void trsv_all(hpb_handle_t h, const hpb_trsv_s* t, const T* val, T alpha, const 
         auto go = [&](auto lprc) {
             hipLaunchKernelGGL((k_trsv_flow<T, COMP, UNIT, decltype(lprc)::value>),
                                dim3((unsigned)flow_waves(t->rows, nl, cus)), dim3(64), 0, st, t->rows, t->recs, t->ci,
-                               val, alpha, b, x, w, next);
+                               val, alpha, b, x, w, next, h->flow_spins, &host_flag_of(h)->flow_gave_up);
         };
         if (COMP || t->lpr == 1) go(std::integral_constant<int, 1>{});
         else if (t->lpr == 2) go(std::integral_constant<int, 2>{});
@@ -386,6 +391,7 @@ int trsv_entry(hpb_handle_t h, hpb_trsv_t t, const T* val, T alpha, const T* b, 
 {
     HPB_CLEAR_STALE();
     HPB_REQUIRE(h && t && val && b && x, HPB_ERR_INVALID, "hpb_csr_trsv: null argument");
+    if (const int rc = flow_status(h)) return rc;   // an earlier solve's
     switch (t->uplo) {
     case 0:
         if (comp) trsv_all<T, true, false, true>(h, t, val, alpha, b, x);

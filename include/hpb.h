@@ -376,6 +376,11 @@ int hpb_csr_trsv_analysis(hpb_handle_t h, int uplo, int rows, int64_t nnz, const
 int hpb_csr_trsv_levels(hpb_trsv_t t, int* nlevels);
 /* kernel launches of a solve: 2 (its workspace and all levels), or one per level */
 int hpb_csr_trsv_launches(hpb_trsv_t t, int* launches);
+/* The rows of a one-launch solve poll for the values they need.  After `polls` polls for
+ * its 64 rows (2^22, seconds, by default) a wave takes NaN for the values that are missing
+ * and the handle remembers it: its next hpb_synchronize, hpb_memcpy_d2h, blocking
+ * reduction or triangular solve returns HPB_ERR_UNSUPPORTED, once. */
+int hpb_set_trsv_wait_limit(hpb_handle_t h, uint32_t polls);
 int hpb_trsv_destroy(hpb_trsv_t t);
 int hpb_csr_trsv_f64(hpb_handle_t h, hpb_trsv_t t, const double* val, double alpha, const double* b, double* x,
                      int compensated);

@@ -339,3 +339,40 @@ def test_where_one_launch_is_taken(handle, deps, nlev, width, one):
     assert launches.value == (2 if one else nlev)
     for a in (rp, ci, va):
         a.free()
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_waits_given_up_are_reported(handle, dtype):
+    """With no polls allowed, the rows of a tridiagonal solve do not find the value of the
+    row before: they hold NaN and the next call that waits says so, once, whichever it is;
+    with the default limit the same solve is right again."""
+    suf, c = ("f64", ctypes.c_double) if dtype == np.float64 else ("f32", ctypes.c_float)
+    n = 500
+    M = sp.diags([np.full(n - 1, -1.0), np.full(n, 4.0)], [-1, 0])
+    rp, ci, va, Ms = _dev_csr(handle, M, dtype)
+    b = np.ones(n, dtype)
+    db, dx = H.DeviceArray.from_numpy(b, handle), H.DeviceArray(n, dtype, handle)
+    t = _analysis(handle, 2, Ms, rp, ci)
+
+    def solve():
+        H.call("hpb_csr_trsv_" + suf, handle.ptr, t, va.ptr, c(1.0), db.ptr, dx.ptr, 0)
+    waiting = (handle.sync, dx.numpy, lambda: H.nrm2c(handle, db), solve)
+    try:
+        for wait in waiting:
+            say("gave up", suf)
+            H.call("hpb_set_trsv_wait_limit", handle.ptr, 0)
+            H.call("hpb_timer_start", handle.ptr)
+            solve()
+            H.call("hpb_set_trsv_wait_limit", handle.ptr, 1 << 22)
+            H.call("hpb_timer_stop", handle.ptr, ctypes.byref(ctypes.c_float()))   # waits, reports nothing
+            with pytest.raises(H.HPBError, match="in vain"):
+                wait()
+            assert np.isnan(dx.numpy()[1:]).any()
+            solve()
+            ref = spla.spsolve_triangular(Ms.astype(np.float64).tocsr(), b.astype(np.float64), lower=True)
+            assert np.max(np.abs(dx.numpy() - ref)) <= (1e-15 if dtype == np.float64 else 1e-6)
+    finally:
+        H.call("hpb_set_trsv_wait_limit", handle.ptr, 1 << 22)
+        H.call("hpb_trsv_destroy", t)
+        for a in (rp, ci, va, db, dx):
+            a.free()
