@@ -340,3 +340,32 @@ def test_spmv_staged_long_rows_bitexact(handle, lpr, n, mean):
     dx = H.DeviceArray.from_numpy(x, handle)
     assert spmv(handle, A, dx, comp=True).numpy().tobytes() == O.csr_spmv(Mh, x, lpr=lpr, comp=True).tobytes()
     A.free()
+
+
+@pytest.mark.parametrize("comp", [False, True])
+@pytest.mark.parametrize("mean,n", [(7, 20011), (24, 200003)])
+def test_spmv_staged_rows_pass_on_infinities_and_nan(handle, mean, n, comp):
+    """Inf and NaN in x reach the rows that hold an entry there, and no others (staged tiles
+    repeat their last entry), the other rows keep the oracle's bits: tiles of 2 lanes and
+    the wide ones."""
+    say("spmv non-finite", mean, comp)
+    r = np.random.default_rng(mean)
+    deg = np.minimum(np.exp(r.normal(np.log(mean / 1.05), 0.5, n)).astype(np.int64) + 1, 300)
+    row = np.repeat(np.arange(n), deg)
+    rp = np.concatenate([[0], np.cumsum(deg)])
+    col = (row + r.integers(-3000, 3000, row.size)) % n
+    Mh = sp.csr_matrix((r.standard_normal(row.size), col.astype(np.int32), rp.astype(np.int32)), shape=(n, n))
+    assert mean == 7 or Mh.nnz >= 4000000
+    x = r.standard_normal(n)
+    x[r.choice(n, 40, replace=False)] = np.tile([np.inf, -np.inf, np.nan, np.inf], 10)
+    x[Mh.indices[-1]] = np.nan   # the entry that the last tile repeats
+    with np.errstate(all="ignore"):
+        want = O.csr_spmv(Mh, x, lpr=default_lpr(Mh), comp=comp)
+    A = upload_csr(handle, Mh)
+    dx = H.DeviceArray.from_numpy(x, handle)
+    y = spmv(handle, A, dx, comp=comp).numpy()
+    ok = np.isfinite(want)
+    assert 0.9 < ok.mean() < 1.0 and np.array_equal(np.isnan(want), np.isnan(y))
+    keep = ~np.isnan(want)
+    assert want[keep].tobytes() == y[keep].tobytes()
+    A.free()

@@ -376,3 +376,64 @@ def test_waits_given_up_are_reported(handle, dtype):
         H.call("hpb_trsv_destroy", t)
         for a in (rp, ci, va, db, dx):
             a.free()
+
+
+def test_captured_solves(handle):
+    """A captured one-launch solve keeps its workspace when a larger pattern makes the
+    handle's grow, and a handle without a workspace captures the launches per level: every
+    replay, with eager work in between, gives the eager solve's bits."""
+    hip = H.lib()
+    n, big = 900, 40000
+    M = sp.diags([np.full(n - 30, -0.3), np.full(n - 1, -1.0), np.full(n, 4.0)], [-30, -1, 0])
+    rp, ci, va, Ms = _dev_csr(handle, M)
+    rb, cb, vb, Mb = _dev_csr(handle, sp.diags([np.full(big - 1, -1.0), np.full(big, 4.0)], [-1, 0]))
+    b = np.random.default_rng(3).standard_normal(n)
+    streams, handles, graphs, arrays = [], [], [], [rp, ci, va, rb, cb, vb]
+    try:
+        for _ in range(2):
+            streams.append(ctypes.c_void_p())
+            assert hip.hipStreamCreate(ctypes.byref(streams[-1])) == 0
+            handles.append(H.Handle(streams[-1]))
+        t = _analysis(handles[0], 2, Ms, rp, ci)
+        db, dx = H.DeviceArray.from_numpy(b, handle), H.DeviceArray(n, np.float64, handle)
+        bb, xb = H.DeviceArray.from_numpy(np.ones(big), handle), H.DeviceArray(big, np.float64, handle)
+        arrays += [db, dx, bb, xb]
+
+        def solve(h):
+            H.call("hpb_csr_trsv_f64", h.ptr, t, va.ptr, ctypes.c_double(1.0), db.ptr, dx.ptr, 0)
+        solve(handles[0])
+        handles[0].sync()
+        want = dx.numpy()
+        for h, st in zip(handles, streams):
+            say("capture", st.value)
+            g, e = ctypes.c_void_p(), ctypes.c_void_p()
+            assert hip.hipStreamBeginCapture(st, 1) == 0   # thread local
+            solve(h)
+            assert hip.hipStreamEndCapture(st, ctypes.byref(g)) == 0
+            nodes = ctypes.c_size_t()
+            assert hip.hipGraphGetNodes(g, None, ctypes.byref(nodes)) == 0
+            assert nodes.value == (2 if h is handles[0] else n)   # every row is a level
+            assert hip.hipGraphInstantiate(ctypes.byref(e), g, None, None, ctypes.c_ulonglong(0)) == 0
+            graphs.append((g, e))
+        tb = _analysis(handles[0], 2, Mb, rb, cb)   # the workspace grows
+        for _ in range(3):
+            for (g, e), h, st in zip(graphs, handles, streams):
+                H.call("hpb_csr_trsv_f64", handles[0].ptr, tb, vb.ptr, ctypes.c_double(1.0), bb.ptr, xb.ptr, 0)
+                handles[0].sync()
+                dx.upload(np.zeros(n))
+                assert hip.hipGraphLaunch(e, st) == 0
+                h.sync()
+                assert dx.numpy().tobytes() == want.tobytes()
+        assert np.max(np.abs(Mb @ xb.numpy() - 1.0)) <= 1e-14
+        H.call("hpb_trsv_destroy", t)
+        H.call("hpb_trsv_destroy", tb)
+    finally:
+        for g, e in graphs:
+            hip.hipGraphExecDestroy(e)
+            hip.hipGraphDestroy(g)
+        for h in handles:
+            h.close()
+        for st in streams:
+            hip.hipStreamDestroy(st)
+        for a in arrays:
+            a.free()
