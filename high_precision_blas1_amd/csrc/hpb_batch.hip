@@ -80,7 +80,6 @@ struct batch_t {
     int* iters = nullptr;           // nsys
     int* nactive = nullptr;         // 1
     double* part = nullptr;         // ntiles * BQ * 2
-    double* dots = nullptr;         // nsys * BQ
     int* hcount = nullptr;          // pinned
     int* tile_list = nullptr;       // ntiles: indices of the tiles of active systems
     int* tile_count = nullptr;      // 1: entries of tile_list in use
@@ -960,7 +959,7 @@ static int free_batch(batch_t* B)
     if (B->exec2) (void)hipGraphExecDestroy(B->exec2);
     if (B->graph2) (void)hipGraphDestroy(B->graph2);
     void* ptrs[] = {B->d_tiles, B->d_tile_first, B->d_row_off, B->rp, B->col, B->val, B->st, B->active,
-                    B->iters, B->nactive, B->part, B->dots, B->tile_list, B->tile_count, B->dinv, B->sd_val,
+                    B->iters, B->nactive, B->part, B->tile_list, B->tile_count, B->dinv, B->sd_val,
                     B->sd_mask, B->sd_off, B->stale, B->confirm, B->bar};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
@@ -1142,7 +1141,6 @@ int hpb_batch_create_diffusion2d(hpb_handle_t h, int nsys, const int* sides, dou
     M((void**)&B->iters, sizeof(int) * nsys);
     M((void**)&B->nactive, sizeof(int));
     M((void**)&B->part, sizeof(double) * 2 * BQ * B->ntiles);
-    M((void**)&B->dots, sizeof(double) * BQ * nsys);
     M((void**)&B->tile_list, sizeof(int) * B->ntiles);
     M((void**)&B->tile_count, sizeof(int));
     M((void**)&B->dinv, sizeof(double) * B->nrows);
