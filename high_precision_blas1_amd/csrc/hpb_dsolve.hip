@@ -1798,6 +1798,7 @@ private:
     // by their launch in either form, and a solve to a loose tolerance may end after a few:
     // four products per digit are counted on.  Whole solves on rows of 5 to 32 diagonals,
     // sliced against CSR, BiCGStab(2):
+    //   to 1e-12, plain, 7 diagonals: 22 k rows +6 %, 27 k +5, 32 k +3, 37 k -2, 45 k -3;
     //   to 1e-10, plain: 33 k rows -3 to +7 %, 50 k -12 to -3, 100 k -20 to -4, 1 M -48 to -11;
     //   compensated: 33 k -3 to +18 %, 70 k -11 to +3, 100 k -14 to +2 (7 diagonals), 150 k
     //     -18 to -5;
@@ -1807,8 +1808,8 @@ private:
     {
         const double each = prm.solver == HPB_SOLVER_GMRES ? 1.0 : 2.0;   // products per iteration
         const double products = std::min(-4.0 * std::log10(std::max(target, 1e-16)), each * prm.max_iters);
-        const double weight = prm.compensated_spmv ? 0.5 : 1.0;
-        return products >= 12.0 && weight * P.rows >= 49152.0 && weight * P.rows * products >= 1.2e6;
+        const double rows = P.rows, least = prm.compensated_spmv ? 98304.0 : 34816.0;
+        return products >= 12.0 && rows >= least && rows * products >= 1.2e6 * (least / 34816.0);
     }
 
     // Decides on the sliced-diagonal form of the matrix (hpb_sdia.hpp): A.K > 0 when it
